@@ -233,3 +233,46 @@ def test_mgpcg_manufactured_solution_second_order(cuda):
         errs.append(np.linalg.norm((v - u)[G]) / np.sqrt(G.sum()))
     ratios = [errs[i] / errs[i + 1] for i in range(2)]
     assert all(3.6 < r < 4.4 for r in ratios), (errs, ratios)
+
+
+# Row lengths around the multiples of eight (four positions per lane of each
+# colour), of 64 (a restriction block's fine columns) and of the 8^3 boxes of
+# the coarsest level; the shortest rows; one to three levels.
+@pytest.mark.parametrize("shape,nlevels", [((1, 1, 1), 1), ((2, 3, 5), 1), ((9, 8, 7), 1),
+                                           ((5, 40, 3), 2), ((62, 9, 10), 2), ((63, 10, 9), 2),
+                                           ((64, 11, 18), 2), ((65, 8, 17), 2), ((66, 18, 16), 2),
+                                           ((33, 35, 34), 2), ((129, 12, 13), 3), ((36, 34, 30), 3)])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_mgpcg_row_lengths(cuda, shape, nlevels, dt):
+    rng = np.random.default_rng(shape[0])
+    m = np.asfortranarray(rng.random(shape) < 0.97)
+    m[shape[0] // 2, shape[1] // 2, shape[2] // 2] = True
+    f = np.asfortranarray((rng.standard_normal(shape) * m).astype(dt))
+    vsz = (0.9, 1.0, 1.3)
+    tol = 1e-12 if dt == np.float64 else 1e-5
+    v, (it, _) = uw.mgpcg(f, m, vsz, tol, 300, {"nlevels": nlevels, "npre": 2, "npost": 2},
+                          return_info=True)
+    assert it < 300
+    assert np.all(v[~m] == 0)
+    # the residual's bound times the condition number, below 1e4 on these grids
+    assert rel_l2(v, po.solve(f, m, vsz)) < (1e-8 if dt == np.float64 else 1e-3)
+    again = uw.mgpcg(f, m, vsz, tol, 300, {"nlevels": nlevels, "npre": 2, "npost": 2})
+    np.testing.assert_array_equal(again, v)
+
+
+@pytest.mark.parametrize("dt", ["float64", "float32"])
+def test_unwrap_work_space_at_any_address(cuda, dt):
+    """The device form's work space may start at any byte."""
+    import torch
+
+    shape = (21, 18, 20)
+    t = torch.rand(shape[::-1], device="cuda", dtype=getattr(torch, dt)).permute(2, 1, 0) * 6 - 3
+    m = torch.ones(shape[::-1], device="cuda", dtype=torch.uint8).permute(2, 1, 0)
+    n = uw.work_bytes(t.dtype, shape)
+    buf = torch.full((n + 64,), 255, dtype=torch.uint8, device="cuda")
+    got = []
+    for off in (0, 1, 24):
+        up, d2 = torch.empty_like(t), torch.empty_like(t)
+        uw.unwrap_laplacian_dev(t, m, (1, 1, 1), up, d2, work=buf[off:off + n])
+        got.append(up)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
