@@ -174,3 +174,32 @@ def test_tv_register_pass_lengths(cuda, dt, shape):
         np.testing.assert_array_equal(gtr[:, 4], wtr[:, 4])
     else:
         assert rel_l2(got, want) < 1e-3
+
+
+# Rows of one group, of a few and of many (a row's end meets its start through
+# the periodic neighbours), nx a multiple of 2 but not of 4, odd nx.
+@pytest.mark.parametrize("shape", [(4, 3, 2), (8, 1, 5), (6, 7, 4), (12, 10, 1), (20, 11, 13),
+                                   (66, 6, 5), (15, 8, 6), (260, 4, 3)])
+@pytest.mark.parametrize("dt", ["float64", "float32"])
+def test_tv_wide_rows_equal_the_voxel_kernels(cuda, shape, dt):
+    """The update and the right-hand side take several voxels per lane where
+    the work space lies on 16 bytes, one otherwise: the same x bit for bit."""
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(shape[0])
+    tdt = getattr(torch, dt)
+    f = torch.randn(shape[::-1], generator=g, device="cuda", dtype=tdt).permute(2, 1, 0)
+    m = (torch.rand(shape[::-1], generator=g, device="cuda") < 0.8).to(torch.uint8).permute(2, 1, 0)
+    n = gtv.work_bytes(tdt, shape)
+    buf = torch.full((n + 16,), 255, dtype=torch.uint8, device="cuda")
+    got = []
+    for off in (0, 8):
+        out = torch.empty_like(f)
+        gtv.tv_dev(f, m, (1.0, 0.9, 1.2), (0.0, 0.1, 0.99),
+                   {"verbose": 0, "maxit": 7, "rtol": 0.0, "atol": 0.0}, out,
+                   work=buf[off:off + n])
+        torch.cuda.synchronize()
+        got.append(out)
+    assert torch.isfinite(got[0]).all()
+    assert torch.equal(got[0], got[1])
