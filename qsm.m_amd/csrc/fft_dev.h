@@ -325,10 +325,21 @@ __device__ __forceinline__ Cx<T> *stockham(Cx<T> *A, Cx<T> *B, Pen pn,
 
 // Where the real volume (nx, ny, nz) sits in the transform grid: offsets
 // (o0, o1, o2) of zero padding before it; H = M0/2 + 1 half-spectrum
-// columns; M1 the y length.
+// columns; M1, M2 the y and z lengths.  On a forward transform the volume
+// may run past the end of y and z and go on at 0 (o1 + ny > M1, o2 + nz >
+// M2): an image centred on sample 0.
 struct RealGeom {
-    int nx, ny, nz, o0, o1, o2, H, M1;
+    int nx, ny, nz, o0, o1, o2, H, M1, M2;
 };
+
+// Index i of an axis of length M that a range may have run past.
+__device__ __forceinline__ int wrap(int i, int M) { return i < M ? i : i - M; }
+
+// Whether index i lies in [lo, hi), a range that runs past M to go on at 0.
+__device__ __forceinline__ bool in_range(int i, int lo, int hi, int M)
+{
+    return (i >= lo && i < hi) || i < hi - M;
+}
 
 }  // namespace fft
 }  // namespace qsm
@@ -513,10 +524,11 @@ __global__ __launch_bounds__(FFT_THREADS) void rx_fwd(
         // 2A = z + conj(w), 2B = -i (z - conj(w))
         const Cx<T> sa{z.re + w.re, z.im - w.im};
         const Cx<T> sb{z.im + w.im, w.re - z.re};
-        const int ja = ra % g.ny + g.o1, ka = ra / g.ny + g.o2;
+        const int ja = wrap(ra % g.ny + g.o1, g.M1), ka = wrap(ra / g.ny + g.o2, g.M2);
         data[size_t(k) + size_t(H) * (size_t(ja) + size_t(g.M1) * ka)] = sa;
         if (ra + 1 < rows) {
-            const int jb = (ra + 1) % g.ny + g.o1, kb = (ra + 1) / g.ny + g.o2;
+            const int jb = wrap((ra + 1) % g.ny + g.o1, g.M1);
+            const int kb = wrap((ra + 1) / g.ny + g.o2, g.M2);
             data[size_t(k) + size_t(H) * (size_t(jb) + size_t(g.M1) * kb)] = sb;
         }
     }
@@ -540,14 +552,14 @@ __global__ __launch_bounds__(FFT_THREADS) void cy_pass(
     const int nxb = (v.M0 + P - 1) / P;
     const int lb = xcd_block();  // neighbouring x groups share L2 lines
     const int x0 = (lb % nxb) * P;
-    const int k = k0 + lb / nxb;
+    const int k = wrap(k0 + lb / nxb, v.M2);
     const int np = min(P, v.M0 - x0);
     const size_t base = size_t(x0) + size_t(k) * v.M0 * v.M1;
     const int logP = pn.logP;
     fill(A, P * M, [&](int e, int &d) {
         const int i = e >> logP, p = e & (P - 1);
         d = i * PP + p;
-        return (p < np && i >= ylo && i < yhi) ? data[base + p + size_t(i) * v.M0]
+        return (p < np && in_range(i, ylo, yhi, M)) ? data[base + p + size_t(i) * v.M0]
                                                : Cx<T>{T(0), T(0)};
     });
     __syncthreads();
@@ -588,7 +600,7 @@ __global__ __launch_bounds__(FFT_THREADS) void z_pass(
     fill(A, P * M, [&](int e, int &d) {
         const int i = e >> logP, p = e & (P - 1);
         d = i * PP + p;
-        return (p < np && i >= zlo && i < zhi) ? data[base + p + size_t(i) * plane]
+        return (p < np && in_range(i, zlo, zhi, M)) ? data[base + p + size_t(i) * plane]
                                                : Cx<T>{T(0), T(0)};
     });
     __syncthreads();
@@ -865,7 +877,7 @@ int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const 
     const int H = M0 / 2 + 1;
     const Vol v{H, M1, M2};  // the volume the y and z passes see
     const RealGeom g{int(sz[0]), int(sz[1]), int(sz[2]), int(off[0]), int(off[1]), int(off[2]),
-                     H, M1};
+                     H, M1, M2};
     const int ny = g.ny, nz = g.nz;
     const size_t cs = sizeof(Cx<T>);
     hipError_t e = hipSuccess;
@@ -879,8 +891,12 @@ int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const 
             work, in, g, pn, ap[0].dpl, tw_of<T>(ap[0]), skip);
         QSM_HIP(hipGetLastError());
     }
+    // the register-resident y and z passes take no range that wraps
+    const bool wy = g.o1 + ny > M1, wz = g.o2 + nz > M2;
+    if (wy || wz)
+        QSM_ARG(!ROUND, "only a forward transform may wrap");
     // y forward on data planes
-    if (y_reg<T>(work, v, g.o2, nz, ap[1], true, g.o1, g.o1 + ny, skip, st, e)) {
+    if (!wy && !wz && y_reg<T>(work, v, g.o2, nz, ap[1], true, g.o1, g.o1 + ny, skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pny = pencils(M1, cs);
@@ -891,7 +907,7 @@ int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const 
     }
     // z forward, op (, z inverse)
     constexpr int ZM = ROUND ? (reg::FWD | reg::OP | reg::INV) : (reg::FWD | reg::OP);
-    if (z_reg<T, ZM>(work, work, v, ap[2], g.o2, g.o2 + nz, op, skip, st, e)) {
+    if (!wz && z_reg<T, ZM>(work, work, v, ap[2], g.o2, g.o2 + nz, op, skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pn = pencils(M2, cs);
@@ -923,7 +939,7 @@ int real_conv_from(const Cx<T> *S, T *out, const size_t sz[3], const size_t M[3]
     const int H = M0 / 2 + 1;
     const Vol v{H, M1, M2};
     const RealGeom g{int(sz[0]), int(sz[1]), int(sz[2]), int(off[0]), int(off[1]), int(off[2]),
-                     H, M1};
+                     H, M1, M2};
     const size_t cs = sizeof(Cx<T>);
     hipError_t e = hipSuccess;
     if (z_reg<T, reg::LOAD_K | reg::OP | reg::INV>(work, S, v, ap[2], g.o2, g.o2 + g.nz, op,

@@ -433,8 +433,9 @@ __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void rx_fwd_reg(
     if (ra >= rows)
         return;
     const int H = g.H;
-    const int ja = ra % g.ny + g.o1, ka = ra / g.ny + g.o2;
-    const int jb = (ra + 1) % g.ny + g.o1, kb = (ra + 1) / g.ny + g.o2;
+    const int ja = wrap(ra % g.ny + g.o1, g.M1), ka = wrap(ra / g.ny + g.o2, g.M2);
+    const int jb = wrap((ra + 1) % g.ny + g.o1, g.M1);
+    const int kb = wrap((ra + 1) / g.ny + g.o2, g.M2);
     Cx<T> *oa = data + size_t(H) * (size_t(ja) + size_t(g.M1) * ka);
     Cx<T> *ob = data + size_t(H) * (size_t(jb) + size_t(g.M1) * kb);
     for (int k = m; k < H; k += TM) {

@@ -138,3 +138,29 @@ def test_empty_mask_gives_zeros(cuda, dt):
             fl, mo = fn(np.asfortranarray(a))
             assert fl.shape == a.shape and fl.dtype == a.dtype and not fl.any()
             assert mo.shape == shape and not mo.any()
+
+
+# The ball's rows and planes wrap around sample 0: axes of 192 samples (the
+# register-resident lengths) in each place, anisotropic voxels with one or
+# two planes on either side, a ball nearly as large as its axis.
+@pytest.mark.parametrize("shape,vsz,r", [((184, 14, 13), (1.0, 1.0, 1.0), 4.0),
+                                         ((13, 184, 14), (1.0, 1.0, 1.0), 4.0),
+                                         ((14, 13, 184), (1.0, 1.0, 1.0), 4.0),
+                                         ((22, 24, 9), (1.0, 1.0, 4.0), 3.0),
+                                         ((21, 16, 14), (2.5, 0.8, 1.7), 3.2),
+                                         ((25, 3, 2), (1.0, 1.0, 1.0), 2.0)])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_ball_wraps_around_sample_zero(cuda, shape, vsz, r, dt):
+    rng = np.random.default_rng(shape[0])
+    f = np.asfortranarray(rng.standard_normal(shape).astype(dt))
+    m = np.ones(shape, bool, order="F")
+    m[0, 0, 0] = False
+    wf, wm = obg.sharp(f, m, vsz, r)
+    gf, gm = gbg.sharp(f, m, vsz, r)
+    np.testing.assert_array_equal(gm, wm)
+    assert rel_l2(gf, wf) < (1e-10 if dt == np.float64 else 1e-4)
+    rs = [r, 0.7 * r]
+    wf, wm = obg.vsharp(f, m, vsz, rs)
+    gf, gm = gbg.vsharp(f, m, vsz, rs)
+    np.testing.assert_array_equal(gm, wm)
+    assert rel_l2(gf, wf) < (1e-10 if dt == np.float64 else 1e-4)
