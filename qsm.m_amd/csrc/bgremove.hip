@@ -127,6 +127,20 @@ __global__ __launch_bounds__(NT) void accumulate_kernel(T *acc, const T *c, cons
     if (l < n) acc[l] = acc[l] + (T(mr[l] ? 1 : 0) - T(mp[l] ? 1 : 0)) * c[l];
 }
 
+// threshold_kernel and accumulate_kernel in one pass: the mask of this radius
+// from its smoothed mask s, and the field's share between it and the last.
+template <typename T>
+__global__ __launch_bounds__(NT) void threshold_accumulate_kernel(uint8_t *mr, const float *s,
+                                                                  T *acc, const T *c,
+                                                                  const uint8_t *mp, size_t n)
+{
+    const size_t l = size_t(blockIdx.x) * NT + threadIdx.x;
+    if (l >= n) return;
+    const uint8_t m = s[l] > 0.999f ? 1 : 0;
+    mr[l] = m;
+    acc[l] = acc[l] + (T(m) - T(mp[l] ? 1 : 0)) * c[l];
+}
+
 template <typename T>
 __global__ __launch_bounds__(NT) void zero_kernel(T *a, size_t n)
 {
@@ -221,18 +235,26 @@ int ball_spectrum(Cx<T> *Sb, T *ball, const size_t M[3], const double vsz[3], do
     return real_conv<T, false>(ball, static_cast<T *>(nullptr), sz, M, off, Sb, KeepOp<T>{}, st);
 }
 
-// The eroded mask of one radius: real(ifft3(H .* fft3(single(mask)))) > 0.999;
+// The smoothed mask of one radius, w.sf = real(ifft3(H .* fft3(single(mask))));
 // from_spectrum: fft3(single(mask)) is already in w.Sm.
+template <typename T>
+int smooth_mask(const Cx<T> *Sb, const size_t szc[3], const size_t M[3], const size_t off[3],
+                Work<T> &w, hipStream_t st, bool from_spectrum = false)
+{
+    SmvOp<T, float, 0> op{Sb, int(M[0] / 2 + 1), int(M[1]),
+                          0.5 / (double(M[0]) * double(M[1]) * double(M[2])), T(0)};
+    Cx<float> *W = reinterpret_cast<Cx<float> *>(w.W);
+    return from_spectrum ? real_conv_from<float>(w.Sm, w.sf, szc, M, off, W, op, st)
+                         : real_conv<float, true>(w.mf, w.sf, szc, M, off, W, op, st);
+}
+
+// The eroded mask of one radius: the smoothed mask > 0.999.
 template <typename T>
 int erode(uint8_t *mout, const Cx<T> *Sb, const size_t szc[3], const size_t M[3],
           const size_t off[3], Work<T> &w, hipStream_t st, bool from_spectrum = false)
 {
     const size_t n = szc[0] * szc[1] * szc[2];
-    SmvOp<T, float, 0> op{Sb, int(M[0] / 2 + 1), int(M[1]),
-                          0.5 / (double(M[0]) * double(M[1]) * double(M[2])), T(0)};
-    Cx<float> *W = reinterpret_cast<Cx<float> *>(w.W);
-    int rc = from_spectrum ? real_conv_from<float>(w.Sm, w.sf, szc, M, off, W, op, st)
-                           : real_conv<float, true>(w.mf, w.sf, szc, M, off, W, op, st);
+    const int rc = smooth_mask<T>(Sb, szc, M, off, w, st, from_spectrum);
     if (rc) return rc;
     threshold_kernel<<<grid1(n), NT, 0, st>>>(mout, w.sf, n);
     QSM_HIP(hipGetLastError());
@@ -308,21 +330,32 @@ int vsharp_t(const T *fc, const uint8_t *mc, const size_t szc[3], size_t nech,
     if (one && (rc = real_conv<T, false>(fc, static_cast<T *>(nullptr), szc, M, off, w.Sf,
                                          KeepOp<T>{}, st)))
         return rc;
+    // the masks of this radius, of the last one and of the one returned, in
+    // three buffers that change places
+    uint8_t *cur = w.m1, *prev = w.mp, *spare = w.mo, *ret = nullptr;
     for (size_t q = 0; q < nrs; ++q) {
         Cx<T> *Sb = q == 0 ? w.Sb1 : w.Sb;  // the first radius's spectrum is kept for ih
         if ((rc = ball_spectrum<T>(Sb, w.ball, M, vsz, rs[q], st))) return rc;
-        if ((rc = erode<T>(w.m1, Sb, szc, M, off, w, st, true))) return rc;
         const SmvOp<T, T, 1> hp{Sb, H, M1, scale, T(thr)};
-        for (size_t e = 0; e < nech; ++e) {
-            rc = one ? real_conv_from<T>(w.Sf, w.c, szc, M, off, w.W, hp, st)
-                     : real_conv<T, true>(fc + e * n, w.c, szc, M, off, w.W, hp, st);
-            if (rc) return rc;
-            accumulate_kernel<T><<<grid1(n), NT, 0, st>>>(flc + e * n, w.c, w.m1, w.mp, n);
+        if (one) {
+            if ((rc = smooth_mask<T>(Sb, szc, M, off, w, st, true))
+                || (rc = real_conv_from<T>(w.Sf, w.c, szc, M, off, w.W, hp, st)))
+                return rc;
+            threshold_accumulate_kernel<T><<<grid1(n), NT, 0, st>>>(cur, w.sf, flc, w.c, prev, n);
             QSM_HIP(hipGetLastError());
+        } else {
+            if ((rc = erode<T>(cur, Sb, szc, M, off, w, st, true))) return rc;
+            for (size_t e = 0; e < nech; ++e) {
+                if ((rc = real_conv<T, true>(fc + e * n, w.c, szc, M, off, w.W, hp, st))) return rc;
+                accumulate_kernel<T><<<grid1(n), NT, 0, st>>>(flc + e * n, w.c, cur, prev, n);
+                QSM_HIP(hipGetLastError());
+            }
         }
-        if (q == qout)
-            QSM_HIP(hipMemcpyAsync(w.mo, w.m1, n, hipMemcpyDeviceToDevice, st));
-        QSM_HIP(hipMemcpyAsync(w.mp, w.m1, n, hipMemcpyDeviceToDevice, st));
+        if (q == qout) ret = cur;
+        // the buffer of the radius before last is free, unless it is returned
+        uint8_t *freed = prev == ret ? spare : prev;
+        prev = cur;
+        cur = freed;
     }
     // f = maskn .* real(ifft3(ih .* fft3(f))), ih from the first radius,
     // maskn the last radius's mask (vsharp.m:142-143)
@@ -330,10 +363,10 @@ int vsharp_t(const T *fc, const uint8_t *mc, const size_t szc[3], size_t nech,
     for (size_t e = 0; e < nech; ++e) {
         T *o = flc + e * n;
         if ((rc = real_conv<T, true>(o, o, szc, M, off, w.W, dc, st))) return rc;
-        mask_kernel<T><<<grid1(n), NT, 0, st>>>(o, w.mp, n);
+        mask_kernel<T><<<grid1(n), NT, 0, st>>>(o, prev, n);
         QSM_HIP(hipGetLastError());
     }
-    QSM_HIP(hipMemcpyAsync(mout, w.mo, n, hipMemcpyDeviceToDevice, st));
+    QSM_HIP(hipMemcpyAsync(mout, ret, n, hipMemcpyDeviceToDevice, st));
     return QSM_OK;
 }
 
