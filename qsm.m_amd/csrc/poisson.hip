@@ -55,7 +55,7 @@ constexpr int DOT_BLOCKS = 1024;  // fixed grid of the dot products
 // pass then reads and writes whole cache lines of what it needs -- one
 // colour of f, the mask and v, the other colour of v -- where the natural
 // order drags both colours of all three through every pass (at 258x258x178
-// padded, FP32: 77 MB against 153 MB).  At equal t a voxel's y and z
+// padded, FP32: 77 MB against 153 MB; a pass 37.4 -> 13.8 us).  At equal t a voxel's y and z
 // neighbours stand at the same t of the other colour, its x neighbours at
 // t - 1 and t (parity 0) or t and t + 1 (parity 1).  Positions past the row's
 // end are zero and their mask bytes clear.
@@ -474,8 +474,9 @@ __device__ __forceinline__ V4<T> lap4(const T *v, size_t p, int colour, int b, u
 // fine box below them go to LDS, four positions at a time and without a
 // barrier in between, then each thread sums its coarse voxels' 27 in the
 // order of restrict_mex.c.  r itself never reaches memory: the separate passes
-// moved 200 MB and took 71 us at 258x258x178 FP32.  (A block that walked the
-// fine planes one by one, a barrier each, took 74 us: latency.)
+// moved 200 MB and took 71 us at 258x258x178 FP32, this one takes 38 us.  (A
+// block that walked the fine planes one by one, a barrier each, took 74 us:
+// latency.)
 constexpr int RX = 32, RY = 4, RZ = 4;
 constexpr int RFY = 2 * RY + 1, RFZ = 2 * RZ + 1;
 constexpr int RG = RX / 4 + 1;  // groups of four per row and colour (the last: one column)
@@ -545,8 +546,9 @@ __global__ __launch_bounds__(NT) void restrict_kernel(T *f2, T *v2, const T *f, 
 // serves the 2x2x2 fine block at (2 i2 - 1, ...)): the mean of the coarse
 // values at the corners the fine voxel lies between (1, 2, 4 or 8 of them).
 // Four positions per lane: they share j, k and the parity of i, so the lanes
-// of a row take the same corners.  Where the mask is clear the coarse values
-// may lie past the row's end (v2 is allocated four positions longer).
+// of a row take the same corners, and a corner row of coarse values is two
+// wide loads (40 -> 31 us at 258x258x178 FP32).  Where the mask is clear the
+// coarse values may lie past the row's end (v2 is allocated four positions longer).
 template <typename T>
 __global__ __launch_bounds__(NT) void correct_kernel(T *v, const T *v2, const uint8_t *G, Dim d,
                                                      Dim d2)
@@ -622,7 +624,8 @@ __global__ __launch_bounds__(NT) void cheb_start_kernel(T *r, T *dn, const T *v,
 // voxel further out, so what is right shrinks by a voxel per step, down to
 // the box.  d and r go to other buffers than they come from (neighbour blocks
 // read the rim); v is needed in the box alone.  One launch per step took
-// about 3 us whatever the level's size: launch and memory latency.
+// about 3 us whatever the level's size, launch and memory latency; one of
+// four steps takes 6.8 us at 34x34x24 FP32, 8.6 us at 43x50x33 FP64.
 constexpr int CS = 4, CB = 8, CR = CB + 2 * CS;
 constexpr int CHEB_NT = CR * CR * CR / 4;
 
