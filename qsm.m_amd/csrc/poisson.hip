@@ -28,9 +28,10 @@
 // operator instead of rounds of 256 Gauss-Seidel sweeps.  Its degree
 // reduces the coarse error by 1e3 over the spectrum bound of the level's
 // box (the masked operator is a principal submatrix of the box's, so the
-// bound holds for any mask); each step is one stencil pass over the level
-// by many workgroups, with no reduction, and a fixed polynomial keeps the
-// V-cycle a fixed linear map, as PCG requires of its preconditioner.
+// bound holds for any mask); its steps are stencil updates by many
+// workgroups, with no reduction, four steps per launch on small levels and
+// one on large ones, and a fixed polynomial keeps the V-cycle a fixed linear
+// map, as PCG requires of its preconditioner.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -594,9 +595,9 @@ __global__ __launch_bounds__(NT) void correct_kernel(T *v, const T *v2, const ui
 // Coarsest level, Chebyshev iteration on hh A (A = -Lap_h, hh = 1 /
 // (2 (hx + hy + hz)), spectrum in [lmin, lmax]; Saad, Iterative Methods for
 // Sparse Linear Systems, 2nd ed., Algorithm 12.1).  Start: r = f - A v on
-// the active voxels, d = s0 hh r with s0 = 1 / theta.
+// the active voxels, d = s0 hh r with s0 = 1 / theta; dz (may be null) = 0.
 template <typename T>
-__global__ __launch_bounds__(NT) void cheb_start_kernel(T *r, T *dn, const T *v, const T *f,
+__global__ __launch_bounds__(NT) void cheb_start_kernel(T *r, T *dn, T *dz, const T *v, const T *f,
                                                         const uint8_t *G, Dim d, Lap c, T s0)
 {
     int col, j, k, b;
@@ -615,19 +616,41 @@ __global__ __launch_bounds__(NT) void cheb_start_kernel(T *r, T *dn, const T *v,
     }
     st4(r + q, o);
     st4(dn + q, dv);
+    if (dz) st4(dz + q, V4<T>{});
 }
 
 // Steps of the iteration: v += d; r -= A d; d = c1 d + c2 hh r (active
-// voxels; d = 0 elsewhere).  A launch takes up to CS steps.  A block owns a
-// CB^3 box and works on it and a rim of CS voxels, on which it holds r in
-// registers and d in LDS, two slots; each step needs its predecessor one
-// voxel further out, so what is right shrinks by a voxel per step, down to
-// the box.  d and r go to other buffers than they come from (neighbour blocks
-// read the rim); v is needed in the box alone.  One launch per step took
-// about 3 us whatever the level's size, launch and memory latency; one of
-// four steps takes 6.8 us at 34x34x24 FP32, 8.6 us at 43x50x33 FP64.
+// voxels; d = 0 elsewhere).
+//
+// Small levels, up to CS steps per launch: a block owns a CB^3 box and works
+// on it and a rim of CS voxels, on which it holds r in registers and d in
+// LDS, two slots; each step needs its predecessor one voxel further out, so
+// what is right shrinks by a voxel per step, down to the box.  d and r go to
+// other buffers than they come from (neighbour blocks read the rim); v is
+// needed in the box alone.  On these levels a launch of one step takes about
+// 3 us whatever the size, launch and memory latency; one of four steps takes
+// 6.8 us at 34x34x24 FP32, 8.6 us at 43x50x33 FP64.
 constexpr int CS = 4, CB = 8, CR = CB + 2 * CS;
 constexpr int CHEB_NT = CR * CR * CR / 4;
+
+dim3 cheb_grid(Dim d)
+{
+    return dim3((d.nx - 2 + CB - 1) / CB, (d.ny - 2 + CB - 1) / CB, (d.nz - 2 + CB - 1) / CB);
+}
+
+// Whether a level takes boxes: those that the chip's 256 CUs hold at once,
+// two per CU in FP32 (32 KB of LDS each) and one in FP64 (64 KB: two fit, but
+// then each takes twice as long).  Solves of one level, one PCG iteration,
+// boxes against one step per launch, MI355X: FP32 0.67 / 0.76 ms at 512 boxes
+// (64x64x64), 0.90 / 0.83 at 648 (72x72x64), 2.76 / 1.46 at 4096 (256x256x30);
+// FP64 0.57 / 0.63 ms at 245 (56x56x40), 0.77 / 0.69 at 294 (56x56x48), 0.94 /
+// 0.97 at 512, 4.59 / 2.75 at 4096.
+template <typename T>
+bool cheb_boxed(Dim d)
+{
+    const dim3 g = cheb_grid(d);
+    return size_t(g.x) * g.y * g.z <= (sizeof(T) == 4 ? 512 : 256);
+}
 
 struct ChebSteps {
     double c1[CS], c2[CS];
@@ -708,6 +731,35 @@ void cheb_steps_kernel(T *v, T *rn, T *dn, const T *r, const T *dd, const uint8_
                 dn[q[e]] = dl[e];
             }
     }
+}
+
+// Large levels, one step per launch, four positions per lane: every field
+// passes through memory once a step, where a box with its rim loads and
+// updates 8 voxels for each of its own.  r is updated in place, d goes to
+// another buffer (its neighbours are read), zero at inactive voxels already.
+template <typename T>
+__global__ __launch_bounds__(NT) void cheb_step_kernel(T *v, T *r, T *dn, const T *dd,
+                                                       const uint8_t *G, Dim d, Lap c, T c1, T c2)
+{
+    int col, j, k, b;
+    size_t p;
+    if (!group4(d, col, j, k, p, b)) return;
+    const size_t q = col * d.half() + p;
+    const uint32_t m = ldm4(G + q);
+    if (m == 0) return;
+    V4<T> dc;
+    const V4<T> la = lap4(dd, p, col, b, m, d, c, dc);
+    V4<T> vv = ld4(v + q), rv = ld4(r + q), o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        // d, r and their Laplacian are zero at an inactive voxel
+        vv.a[e] = vv.a[e] + dc.a[e];
+        rv.a[e] = rv.a[e] + la.a[e];
+        o.a[e] = c1 * dc.a[e] + c2 * T(1.0 / (2.0 * (c.hx + c.hy + c.hz))) * rv.a[e];
+    }
+    st4(v + q, vv);
+    st4(r + q, rv);
+    st4(dn + q, o);
 }
 
 // ---- PCG vector kernels ----------------------------------------------------
@@ -916,7 +968,7 @@ struct Solver {
     int L;
     Level<T> lv[MAX_LEVELS];
     T *x, *p;           // PCG iterate and direction (level-0 size)
-    T *cd[2], *cr[2];   // coarsest level: the Chebyshev d and r, two buffers each
+    T *cd[2], *cr[2];   // coarsest level: the Chebyshev d and r (cr[1]: where boxes update it)
     uint8_t *gn[2];     // masks of a level and the next in natural order (set-up)
     uint8_t *tmp;       // band seed scratch (level-0 size)
     int *rowcnt, *btot; // band list construction: per-row counts, totals per level
@@ -961,7 +1013,8 @@ size_t solver_layout(const size_t sz[3], const double vsz[3], int L, Solver<T> *
     char *pbt = take(2 * MAX_LEVELS * sizeof(int));
     const size_t nc = d[L - 1].n();
     char *pc[4];
-    for (char *&c : pc) c = take(nc * sizeof(T));
+    for (int a = 0; a < 4; ++a)
+        pc[a] = a < 3 || cheb_boxed<T>(d[L - 1]) ? take(nc * sizeof(T)) : nullptr;
     char *ppart = take(DOT_BLOCKS * sizeof(double)), *psum = take(sizeof(double));
     char *ppcg = take(sizeof(Pcg));
     if (s) {
@@ -1067,13 +1120,24 @@ int coarse_solve(Solver<T> &s, Level<T> &L, hipStream_t st)
     const Cheb ch = cheb_of(L.d, L.c);
     const double theta = 0.5 * (ch.lmax + ch.lmin), delta = 0.5 * (ch.lmax - ch.lmin);
     const double sigma = theta / delta;
-    cheb_start_kernel<T><<<grid4(L.d, 2), NT, 0, st>>>(s.cr[0], s.cd[0], L.v, L.f, L.G, L.d, L.c,
-                                                       T(1.0 / theta));
+    const bool boxed = cheb_boxed<T>(L.d);
+    cheb_start_kernel<T><<<grid4(L.d, 2), NT, 0, st>>>(s.cr[0], s.cd[0], boxed ? nullptr : s.cd[1],
+                                                       L.v, L.f, L.G, L.d, L.c, T(1.0 / theta));
     QSM_HIP(hipGetLastError());
-    const dim3 g((L.d.nx - 2 + CB - 1) / CB, (L.d.ny - 2 + CB - 1) / CB,
-                 (L.d.nz - 2 + CB - 1) / CB);
     double rho = 1.0 / sigma;
     int cur = 0;
+    if (!boxed) {
+        for (int k = 0; k < ch.K; ++k, cur ^= 1) {
+            const double rho1 = 1.0 / (2.0 * sigma - rho);
+            cheb_step_kernel<T><<<grid4(L.d, 2), NT, 0, st>>>(
+                L.v, s.cr[0], s.cd[cur ^ 1], s.cd[cur], L.G, L.d, L.c, T(rho1 * rho),
+                T(2.0 * rho1 / delta));
+            QSM_HIP(hipGetLastError());
+            rho = rho1;
+        }
+        return QSM_OK;
+    }
+    const dim3 g = cheb_grid(L.d);
     for (int k = 0; k < ch.K; k += CS) {
         ChebSteps cs;
         cs.n = std::min(CS, ch.K - k);

@@ -276,3 +276,29 @@ def test_unwrap_work_space_at_any_address(cuda, dt):
         uw.unwrap_laplacian_dev(t, m, (1, 1, 1), up, d2, work=buf[off:off + n])
         got.append(up)
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+# One-level solves on either side of the lines between the coarsest level's
+# two kernels (512 boxes of 8^3 in FP32, 256 in FP64), the grid's rows and
+# planes in each place, rows that end within a group of four.  The Chebyshev
+# polynomial maps the spectrum of the operator into 1 +- 1e-3 whatever the
+# mask, so PCG's bound is 2 (5e-4)^k in the energy norm and, with the square
+# root of the condition number below 100, 200 (5e-4)^k in the residual: 5
+# iterations for 1e-12, 3 for 1e-5, one more for rounding.
+@pytest.mark.parametrize("shape", [(128, 128, 1), (129, 128, 1), (128, 256, 1), (129, 256, 1),
+                                   (2, 127, 259), (127, 259, 2), (259, 2, 127), (18, 131, 137),
+                                   (64, 62, 63), (66, 67, 65)])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_mgpcg_coarsest_level_sizes(cuda, shape, dt):
+    rng = np.random.default_rng(shape[0])
+    m = np.asfortranarray(rng.random(shape) < 0.97)
+    m[:, : shape[1] // 4] = False  # whole groups and boxes without a voxel
+    f = np.asfortranarray((rng.standard_normal(shape) * m).astype(dt))
+    vsz = (0.9, 1.0, 1.3)
+    tol, bound = (1e-12, 6) if dt == np.float64 else (1e-5, 4)
+    o = {"nlevels": 1}
+    v, (it, _) = uw.mgpcg(f, m, vsz, tol, 30, o, return_info=True)
+    assert it <= bound
+    assert np.all(v[~m] == 0)
+    assert _true_relres(v, f, m, vsz) < (1e-11 if dt == np.float64 else 1e-4)
+    np.testing.assert_array_equal(uw.mgpcg(f, m, vsz, tol, 30, o), v)
