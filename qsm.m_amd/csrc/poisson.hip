@@ -179,10 +179,13 @@ Lap lap_at(const double vsz[3], int level)
 
 // out = in with a zero border of one voxel; sgn_mask != 0: out = sgn_mask *
 // mask .* in (unwrapLaplacian's -m.*d2u).  One lane per position, those past
-// the row's end included.
+// the row's end included.  G (may be null): the mask with a zero border, in
+// natural order, here and not in a launch of its own: 15 us for both at
+// 258x258x62 FP32 against 11 + 17, and a launch more ahead of the set-up's
+// read-back costs the smallest solves 25 us (set-up alone 68 against 94).
 template <typename T>
-__global__ __launch_bounds__(NT) void pad_kernel(T *out, const T *in, const uint8_t *m, Dim dp,
-                                                 T sgn_mask)
+__global__ __launch_bounds__(NT) void pad_kernel(T *out, const T *in, uint8_t *G, const uint8_t *m,
+                                                 Dim dp, T sgn_mask)
 {
     int c, j, k, b;
     size_t p;
@@ -191,23 +194,14 @@ __global__ __launch_bounds__(NT) void pad_kernel(T *out, const T *in, const uint
     V4<T> v;
     for (int e = 0; e < 4; ++e) {
         const int i = 2 * (t + e) + b;
+        const bool in_box = interior(dp, i, j, k);
+        const size_t li = size_t(i - 1) +
+                          size_t(dp.nx - 2) * (size_t(j - 1) + size_t(dp.ny - 2) * (k - 1));
         v.a[e] = T(0);
-        if (interior(dp, i, j, k)) {
-            const size_t li = size_t(i - 1) +
-                              size_t(dp.nx - 2) * (size_t(j - 1) + size_t(dp.ny - 2) * (k - 1));
-            v.a[e] = (sgn_mask != T(0)) ? sgn_mask * (T(m[li] ? 1 : 0) * in[li]) : in[li];
-        }
+        if (in_box) v.a[e] = (sgn_mask != T(0)) ? sgn_mask * (T(m[li] ? 1 : 0) * in[li]) : in[li];
+        if (G && i < dp.nx) G[nidx(dp, i, j, k)] = in_box && m[li] ? 1 : 0;
     }
     st4(out + c * dp.half() + p, v);
-}
-
-// The mask with a zero border, in natural order.
-__global__ __launch_bounds__(NT) void pad_mask_kernel(uint8_t *G, const uint8_t *m, Dim dp)
-{
-    int i, j, k;
-    if (!vox(dp, i, j, k)) return;
-    const size_t li = size_t(i - 1) + size_t(dp.nx - 2) * (size_t(j - 1) + size_t(dp.ny - 2) * (k - 1));
-    G[nidx(dp, i, j, k)] = interior(dp, i, j, k) ? (m[li] ? 1 : 0) : 0;
 }
 
 template <typename T>
@@ -1211,8 +1205,8 @@ int mgpcg_t(const T *src, bool unwrap, const uint8_t *mask, const size_t sz[3],
     // level 0: r (held in f) = padded right-hand side; masks of the hierarchy
     // (built in natural order, kept split); v zero, which faces and inactive
     // voxels stay (restrict_kernel clears the rest for each cycle)
-    pad_kernel<T><<<grid4(L0.d, 2), NT, 0, st>>>(L0.f, src, mask, L0.d, unwrap ? T(-1) : T(0));
-    pad_mask_kernel<<<grid3(L0.d), b, 0, st>>>(s.gn[0], mask, L0.d);
+    pad_kernel<T><<<grid4(L0.d, 2), NT, 0, st>>>(L0.f, src, s.gn[0], mask, L0.d,
+                                                 unwrap ? T(-1) : T(0));
     QSM_HIP(hipGetLastError());
     for (int l = 0; l < s.L; ++l) {
         Level<T> &L = s.lv[l];
@@ -1254,7 +1248,7 @@ int mgpcg_t(const T *src, bool unwrap, const uint8_t *mask, const size_t sz[3],
     res = std::sqrt(res);
     const double reltol = tol * res;
     if (x0) {
-        pad_kernel<T><<<grid4(L0.d, 2), NT, 0, st>>>(s.x, x0, mask, L0.d, T(0));
+        pad_kernel<T><<<grid4(L0.d, 2), NT, 0, st>>>(s.x, x0, nullptr, mask, L0.d, T(0));
         apply_kernel<T, false><<<DOT_BLOCKS, NT, 0, st>>>(q, s.x, L0.G, L0.d, L0.c, s.part);
         sub_kernel<T><<<g1(n0), NT, 0, st>>>(r, q, n0);
         QSM_HIP(hipGetLastError());
