@@ -754,6 +754,15 @@ size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 constexpr int TPB = 4;
 int tile_grid(int ntiles) { return (ntiles + TPB - 1) / TPB; }
 
+// Grid of the kernels of several voxels per lane: a tile there is 1024 voxels
+// (FP64: 512), and blocks that walk four of them leave CUs idle on small
+// volumes, so there are at least four blocks per CU while there are tiles for
+// them.  20 iterations of tv.m, MI355X, voxel kernels / four tiles per block /
+// this grid: FP32 1.05 / 1.11 / 0.93 ms at 32^3, 1.23 / 1.29 / 1.13 at 64^3,
+// 1.61 / 1.63 / 1.53 at 96x100x80, 2.47 / 2.23 / 2.22 at 128^3; FP64 1.21 / 1.20 /
+// 1.06 at 32^3; the same above (1024 against 512 or 2048 blocks: within 2 %).
+int wide_grid(int ntiles) { return std::max(tile_grid(ntiles), std::min(ntiles, 1024)); }
+
 template <typename T>
 size_t work_layout(const size_t sz[3], Work<T> *w, char *base, bool lsmr = false)
 {
@@ -891,7 +900,7 @@ int admm_run(const T *src, const uint8_t *mask, const size_t sz[3], const double
     const int rgrid = tile_grid(nblk), ugrid = rgrid;
     // the work space's volumes are 256 bytes apart, so one address tells
     const bool wide = o.tv == 1 && g.nx % VW<T> == 0 && reinterpret_cast<uintptr_t>(w.r) % 16 == 0;
-    const int ngrp = int(N) / VW<T>, wgrid = tile_grid((ngrp + NT - 1) / NT);
+    const int ngrp = int(N) / VW<T>, wgrid = wide_grid((ngrp + NT - 1) / NT);
 
     // (v, l) alternate between the two sets: the update reads one, writes
     // the other.  Once the rule stops the loop every later launch returns

@@ -203,3 +203,36 @@ def test_tv_wide_rows_equal_the_voxel_kernels(cuda, shape, dt):
         got.append(out)
     assert torch.isfinite(got[0]).all()
     assert torch.equal(got[0], got[1])
+
+
+# Grids of the wide kernels: one tile (1024 voxels FP32, 512 FP64) and less,
+# up to 1024 blocks of one tile, 1024 blocks that walk two to four, more.
+@pytest.mark.parametrize("shape", [(4, 4, 4), (16, 16, 5), (64, 128, 64), (64, 128, 65),
+                                   (64, 128, 128), (64, 128, 130), (132, 126, 250),
+                                   (132, 126, 260)])
+@pytest.mark.parametrize("dt", ["float64", "float32"])
+def test_tv_wide_grids_equal_the_voxel_kernels(cuda, shape, dt):
+    """x bit for bit and the rule's sums (doubles of one sign in another
+    order, each through fewer than 100 additions, so within 2e-14) through
+    iterations that keep and that change rho."""
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(shape[2])
+    tdt = getattr(torch, dt)
+    f = torch.randn(shape[::-1], generator=g, device="cuda", dtype=tdt).permute(2, 1, 0)
+    m = torch.ones(shape[::-1], dtype=torch.uint8, device="cuda").permute(2, 1, 0)
+    n = gtv.work_bytes(tdt, shape)
+    buf = torch.full((n + 16,), 255, dtype=torch.uint8, device="cuda")
+    got, traces = [], []
+    for off in (0, 8):
+        out, tr = torch.empty_like(f), np.zeros(5 * 7)
+        gtv.tv_dev(f, m, (1.0, 0.9, 1.2), (0.0, 0.1, 0.99),
+                   {"verbose": 0, "maxit": 7, "rtol": 0.0, "atol": 0.0}, out,
+                   work=buf[off:off + n], trace=tr)
+        torch.cuda.synchronize()
+        got.append(out)
+        traces.append(tr.reshape(7, 5))
+    assert torch.equal(got[0], got[1])
+    np.testing.assert_allclose(traces[0], traces[1], rtol=1e-13, atol=0)
+    assert np.unique(traces[0][:, 4]).size > 1
