@@ -340,16 +340,16 @@ __global__ __launch_bounds__(NT) void update_kernel(CVec3<T> v, CVec3<T> lm, Vec
 
 // ---- several voxels per lane -----------------------------------------------
 //
-// The update reads 22 and writes 7 values per voxel.  With 4 bytes per lane
-// each of those is a memory instruction of 15-23 CU cycles (all CUs at once)
-// whatever it hits, and the scalar kernel's time was that count: 176 us at
-// 256x256x176 FP32, 3.7 TB/s of the 14 volumes it must move.  Here a lane
-// takes VW consecutive voxels of a row (16 bytes of every volume): 15 wide
-// loads, 5 narrow ones and 7 wide stores per VW voxels, the -x neighbour's
-// update carried from voxel to voxel: 133 us, 4.9 TB/s (FP64 at 180x216x130:
-// 153 -> 117 us).  Taken where the rows are whole groups
-// (nx a multiple of VW) and every volume starts on 16 bytes; anisotropic
-// only, where a neighbour's update needs one component.
+// The update loads 22 values per voxel (19 of its own, u[l] again for three
+// neighbours) and stores 7.  With 4 bytes per lane each of those is a memory
+// instruction of 15-23 CU cycles (all CUs at once) whatever it hits, and the
+// scalar kernel's time was that count: 176 us at 256x256x176 FP32, 3.7 TB/s
+// of the 14 volumes it must move.  Here a lane takes VW consecutive voxels of
+// a row (16 bytes of every volume): 15 wide loads, 4 narrow ones and 7 wide
+// stores per VW voxels, the -x neighbour's update carried from voxel to
+// voxel: 133 us, 4.9 TB/s (FP64 at 180x216x130: 153 -> 117 us).  Taken where
+// the rows are whole groups (nx a multiple of VW) and every volume starts on
+// 16 bytes; anisotropic only, where a neighbour's update needs one component.
 
 template <typename T>
 constexpr int VW = 16 / int(sizeof(T));
