@@ -232,7 +232,8 @@ int ball_spectrum(Cx<T> *Sb, T *ball, const size_t M[3], const double vsz[3], do
         ball, int(M[0]), int(R1), int(R2), vsz[0], vsz[1], vsz[2], r * r, T(1.0 / double(K)));
     QSM_HIP(hipGetLastError());
     const size_t off[3] = {0, R1 > 0 ? M[1] - R1 : 0, R2 > 0 ? M[2] - R2 : 0};
-    return real_conv<T, false>(ball, static_cast<T *>(nullptr), sz, M, off, Sb, KeepOp<T>{}, st);
+    return real_conv<T, false, true>(ball, static_cast<T *>(nullptr), sz, M, off, Sb, KeepOp<T>{},
+                                     st);
 }
 
 // The smoothed mask of one radius, w.sf = real(ifft3(H .* fft3(single(mask))));

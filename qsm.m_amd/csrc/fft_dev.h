@@ -325,20 +325,27 @@ __device__ __forceinline__ Cx<T> *stockham(Cx<T> *A, Cx<T> *B, Pen pn,
 
 // Where the real volume (nx, ny, nz) sits in the transform grid: offsets
 // (o0, o1, o2) of zero padding before it; H = M0/2 + 1 half-spectrum
-// columns; M1, M2 the y and z lengths.  On a forward transform the volume
-// may run past the end of y and z and go on at 0 (o1 + ny > M1, o2 + nz >
-// M2): an image centred on sample 0.
+// columns; M1, M2 the y and z lengths.  In a forward transform compiled with
+// WRAP the volume may run past the end of y and z and go on at 0 (o1 + ny >
+// M1, o2 + nz > M2): an image centred on sample 0.  A template parameter of
+// the passes, as deciding it per element costs every other convolution 1 %
+// (150x150x100 dipole convolution FP32 83.1 -> 83.9 us).
 struct RealGeom {
     int nx, ny, nz, o0, o1, o2, H, M1, M2;
 };
 
-// Index i of an axis of length M that a range may have run past.
-__device__ __forceinline__ int wrap(int i, int M) { return i < M ? i : i - M; }
+// Index i of an axis of length M that a range may have run past (WRAP).
+template <bool WRAP>
+__device__ __forceinline__ int wrap(int i, int M) { return !WRAP || i < M ? i : i - M; }
 
-// Whether index i lies in [lo, hi), a range that runs past M to go on at 0.
+// Whether index i lies in [lo, hi), with WRAP a range that may run past M to
+// go on at 0.
+template <bool WRAP>
 __device__ __forceinline__ bool in_range(int i, int lo, int hi, int M)
 {
-    return (i >= lo && i < hi) || i < hi - M;
+    // no short circuit here or at the calls: one mask and branch per load
+    const bool in = (i >= lo) & (i < hi);
+    return WRAP ? in | (i < hi - M) : in;
 }
 
 }  // namespace fft
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(FFT_THREADS) void pass_kernel(
 // conj(Z(M - k)) the row spectra are A = (Z + W)/2 and B = (Z - W)/(2i).
 // Stored: 2A and 2B for k = 0..H-1 (the caller folds the 1/2 into its
 // scaling) into the half-spectrum volume (H, M1, M2).
-template <typename T>
+template <typename T, bool WRAP = false>
 __global__ __launch_bounds__(FFT_THREADS) void rx_fwd(
     Cx<T> *data, const T *in, RealGeom g, Pen pn, const Plan *pl, const Cx<T> *tw,
     const int *skip)
@@ -524,11 +531,12 @@ __global__ __launch_bounds__(FFT_THREADS) void rx_fwd(
         // 2A = z + conj(w), 2B = -i (z - conj(w))
         const Cx<T> sa{z.re + w.re, z.im - w.im};
         const Cx<T> sb{z.im + w.im, w.re - z.re};
-        const int ja = wrap(ra % g.ny + g.o1, g.M1), ka = wrap(ra / g.ny + g.o2, g.M2);
+        const int ja = wrap<WRAP>(ra % g.ny + g.o1, g.M1);
+        const int ka = wrap<WRAP>(ra / g.ny + g.o2, g.M2);
         data[size_t(k) + size_t(H) * (size_t(ja) + size_t(g.M1) * ka)] = sa;
         if (ra + 1 < rows) {
-            const int jb = wrap((ra + 1) % g.ny + g.o1, g.M1);
-            const int kb = wrap((ra + 1) / g.ny + g.o2, g.M2);
+            const int jb = wrap<WRAP>((ra + 1) % g.ny + g.o1, g.M1);
+            const int kb = wrap<WRAP>((ra + 1) / g.ny + g.o2, g.M2);
             data[size_t(k) + size_t(H) * (size_t(jb) + size_t(g.M1) * kb)] = sb;
         }
     }
@@ -537,7 +545,7 @@ __global__ __launch_bounds__(FFT_THREADS) void rx_fwd(
 // y pass over planes k in [k0, k0 + nk) (forward or inverse).  Rows
 // outside [ylo, yhi) are zero on input (not read); only rows in
 // [slo, shi) are stored (the later passes read no others).
-template <typename T>
+template <typename T, bool WRAP = false>
 __global__ __launch_bounds__(FFT_THREADS) void cy_pass(
     Cx<T> *data, Vol v, int k0, Pen pn, const Plan *pl, const Cx<T> *tw, T sgn,
     int ylo, int yhi, int slo, int shi, const int *skip)
@@ -552,15 +560,15 @@ __global__ __launch_bounds__(FFT_THREADS) void cy_pass(
     const int nxb = (v.M0 + P - 1) / P;
     const int lb = xcd_block();  // neighbouring x groups share L2 lines
     const int x0 = (lb % nxb) * P;
-    const int k = wrap(k0 + lb / nxb, v.M2);
+    const int k = wrap<WRAP>(k0 + lb / nxb, v.M2);
     const int np = min(P, v.M0 - x0);
     const size_t base = size_t(x0) + size_t(k) * v.M0 * v.M1;
     const int logP = pn.logP;
     fill(A, P * M, [&](int e, int &d) {
         const int i = e >> logP, p = e & (P - 1);
         d = i * PP + p;
-        return (p < np && in_range(i, ylo, yhi, M)) ? data[base + p + size_t(i) * v.M0]
-                                               : Cx<T>{T(0), T(0)};
+        const bool on = (p < np) & in_range<WRAP>(i, ylo, yhi, M);
+        return on ? data[base + p + size_t(i) * v.M0] : Cx<T>{T(0), T(0)};
     });
     __syncthreads();
     Cx<T> *R = stockham(A, B, pn, pl, tw, sgn);
@@ -577,7 +585,7 @@ __global__ __launch_bounds__(FFT_THREADS) void cy_pass(
 // transform.  Only planes [zlo, zhi) hold data on input and only they are
 // needed on output (others neither read nor stored); without ROUND every
 // plane of the spectrum is stored.
-template <typename T, bool ROUND, typename Op>
+template <typename T, bool ROUND, bool WRAP, typename Op>
 __global__ __launch_bounds__(FFT_THREADS) void z_pass(
     Cx<T> *data, Vol v, Pen pn, const Plan *pl, const Cx<T> *tw, int zlo, int zhi, Op op,
     const int *skip)
@@ -600,8 +608,8 @@ __global__ __launch_bounds__(FFT_THREADS) void z_pass(
     fill(A, P * M, [&](int e, int &d) {
         const int i = e >> logP, p = e & (P - 1);
         d = i * PP + p;
-        return (p < np && in_range(i, zlo, zhi, M)) ? data[base + p + size_t(i) * plane]
-                                               : Cx<T>{T(0), T(0)};
+        const bool on = (p < np) & in_range<WRAP>(i, zlo, zhi, M);
+        return on ? data[base + p + size_t(i) * plane] : Cx<T>{T(0), T(0)};
     });
     __syncthreads();
     Cx<T> *R = stockham(A, B, pn, pl, tw, T(-1));
@@ -829,7 +837,8 @@ bool z_reg(Cx<T> *dst, const Cx<T> *src, const Vol &v, const AxisPlan &ap, int z
 // result is transformed back without the 1/(M0 M1 M2)); work holds
 // (M0/2 + 1) M1 M2 complex values and needs no clearing.  With
 // ROUND = false the passes stop after op: work then holds op(2 FFT3(pad(in)))
-// on every plane, and out is not touched.  skip (device flag, may be NULL):
+// on every plane, and out is not touched; with WRAP too the volume may run
+// past the end of y and z and go on at 0.  skip (device flag, may be NULL):
 // the passes do nothing when it is set at their turn on the stream.
 // Inverse y pass on the output planes, then the inverse x pass on the
 // output rows (two per transform, cropped into out).
@@ -862,16 +871,20 @@ int inverse_yx(Cx<T> *work, T *out, const RealGeom &g, const Vol &v, const AxisP
     return QSM_OK;
 }
 
-template <typename T, bool ROUND, typename Op>
+template <typename T, bool ROUND, bool WRAP = false, typename Op>
 int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const size_t off[3],
               Cx<T> *work, Op op, hipStream_t st, const int *skip = nullptr)
 {
+    static_assert(!ROUND || !WRAP, "only a forward transform may wrap");
     int rc;
     AxisPlan ap[3];
     for (int a = 0; a < 3; ++a)
         if ((rc = make_axis<T>(ap[a], M[a], "transform length"))) return rc;
-    if ((rc = allow_lds<&rx_fwd<T>>()) || (rc = allow_lds<&cy_pass<T>>())
-        || (rc = allow_lds<&z_pass<T, ROUND, Op>>()) || (rc = allow_lds<&rx_inv<T>>()))
+    QSM_ARG(WRAP || (off[1] + sz[1] <= M[1] && off[2] + sz[2] <= M[2]),
+            "the volume runs past the transform grid");
+    if ((rc = allow_lds<&rx_fwd<T, WRAP>>()) || (rc = allow_lds<&cy_pass<T, WRAP>>())
+        || (rc = allow_lds<&z_pass<T, ROUND, WRAP, Op>>())
+        || (ROUND && ((rc = allow_lds<&cy_pass<T>>()) || (rc = allow_lds<&rx_inv<T>>()))))
         return rc;
     const int M0 = int(M[0]), M1 = int(M[1]), M2 = int(M[2]);
     const int H = M0 / 2 + 1;
@@ -882,37 +895,34 @@ int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const 
     const size_t cs = sizeof(Cx<T>);
     hipError_t e = hipSuccess;
     // x forward on data rows, two per transform
-    if (reg::launch_x<T>(M0, true, work, in, nullptr, g, twM_of<T>(ap[0]), skip, st, e)) {
+    if (reg::launch_x<T, WRAP>(M0, true, work, in, nullptr, g, twM_of<T>(ap[0]), skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pn = pencils(M0, cs);
         const int P2 = 2 << pn.logP;
-        rx_fwd<T><<<(ny * nz + P2 - 1) / P2, FFT_THREADS, lds_bytes(pn, M0, cs), st>>>(
+        rx_fwd<T, WRAP><<<(ny * nz + P2 - 1) / P2, FFT_THREADS, lds_bytes(pn, M0, cs), st>>>(
             work, in, g, pn, ap[0].dpl, tw_of<T>(ap[0]), skip);
         QSM_HIP(hipGetLastError());
     }
-    // the register-resident y and z passes take no range that wraps
-    const bool wy = g.o1 + ny > M1, wz = g.o2 + nz > M2;
-    if (wy || wz)
-        QSM_ARG(!ROUND, "only a forward transform may wrap");
-    // y forward on data planes
-    if (!wy && !wz && y_reg<T>(work, v, g.o2, nz, ap[1], true, g.o1, g.o1 + ny, skip, st, e)) {
+    // y forward on data planes (the register-resident y and z passes take no
+    // range that wraps)
+    if (!WRAP && y_reg<T>(work, v, g.o2, nz, ap[1], true, g.o1, g.o1 + ny, skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pny = pencils(M1, cs);
         const int Py = 1 << pny.logP;
-        cy_pass<T><<<((H + Py - 1) / Py) * nz, FFT_THREADS, lds_bytes(pny, M1, cs), st>>>(
+        cy_pass<T, WRAP><<<((H + Py - 1) / Py) * nz, FFT_THREADS, lds_bytes(pny, M1, cs), st>>>(
             work, v, g.o2, pny, ap[1].dpl, tw_of<T>(ap[1]), T(-1), g.o1, g.o1 + ny, 0, M1, skip);
         QSM_HIP(hipGetLastError());
     }
     // z forward, op (, z inverse)
     constexpr int ZM = ROUND ? (reg::FWD | reg::OP | reg::INV) : (reg::FWD | reg::OP);
-    if (!wz && z_reg<T, ZM>(work, work, v, ap[2], g.o2, g.o2 + nz, op, skip, st, e)) {
+    if (!WRAP && z_reg<T, ZM>(work, work, v, ap[2], g.o2, g.o2 + nz, op, skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pn = pencils(M2, cs);
         const int P = 1 << pn.logP;
-        z_pass<T, ROUND, Op><<<((H + P - 1) / P) * M1, FFT_THREADS, lds_bytes(pn, M2, cs), st>>>(
+        z_pass<T, ROUND, WRAP><<<((H + P - 1) / P) * M1, FFT_THREADS, lds_bytes(pn, M2, cs), st>>>(
             work, v, pn, ap[2].dpl, tw_of<T>(ap[2]), g.o2, g.o2 + nz, op, skip);
         QSM_HIP(hipGetLastError());
     }

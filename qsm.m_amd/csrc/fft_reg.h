@@ -375,7 +375,7 @@ constexpr int xpencils() { return sizeof(T) == 4 ? 8 : 4; }
 // k < H, of the two rows (A = (Z(k) + conj Z(M-k))/2, B = (Z(k) - conj
 // Z(M-k))/2i with Z the spectrum of the packed pencil), as the Stockham
 // rx_fwd stores them.
-template <typename T, int N1, int N2, int P>
+template <typename T, int N1, int N2, int P, bool WRAP>
 __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void rx_fwd_reg(
     Cx<T> *data, const T *in, RealGeom g, const Cx<T> *twM, const int *skip)
 {
@@ -433,9 +433,9 @@ __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void rx_fwd_reg(
     if (ra >= rows)
         return;
     const int H = g.H;
-    const int ja = wrap(ra % g.ny + g.o1, g.M1), ka = wrap(ra / g.ny + g.o2, g.M2);
-    const int jb = wrap((ra + 1) % g.ny + g.o1, g.M1);
-    const int kb = wrap((ra + 1) / g.ny + g.o2, g.M2);
+    const int ja = wrap<WRAP>(ra % g.ny + g.o1, g.M1), ka = wrap<WRAP>(ra / g.ny + g.o2, g.M2);
+    const int jb = wrap<WRAP>((ra + 1) % g.ny + g.o1, g.M1);
+    const int kb = wrap<WRAP>((ra + 1) / g.ny + g.o2, g.M2);
     Cx<T> *oa = data + size_t(H) * (size_t(ja) + size_t(g.M1) * ka);
     Cx<T> *ob = data + size_t(H) * (size_t(jb) + size_t(g.M1) * kb);
     for (int k = m; k < H; k += TM) {
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void rx_inv_reg(
     }
 }
 
-template <typename T, int N1, int N2>
+template <typename T, int N1, int N2, bool WRAP>
 hipError_t launch_x_one(bool forward, Cx<T> *data, const T *in, T *out, const RealGeom &g,
                         const Cx<T> *twM, const int *skip, hipStream_t st)
 {
@@ -529,28 +529,35 @@ hipError_t launch_x_one(bool forward, Cx<T> *data, const T *in, T *out, const Re
     const int nblk = (rows + 2 * P - 1) / (2 * P);
     if (nblk > 0) {
         if (forward)
-            rx_fwd_reg<T, N1, N2, P><<<nblk, NT, 0, st>>>(data, in, g, twM, skip);
+            rx_fwd_reg<T, N1, N2, P, WRAP><<<nblk, NT, 0, st>>>(data, in, g, twM, skip);
         else
             rx_inv_reg<T, N1, N2, P><<<nblk, NT, 0, st>>>(data, out, g, twM, skip);
     }
     return hipGetLastError();
 }
 
+template <int N>
+using Len = std::integral_constant<int, N>;
+
 // The x pass of length M in the register form; false when M has no split.
-template <typename T>
+template <typename T, bool WRAP = false>
 bool launch_x(int M, bool forward, Cx<T> *data, const T *in, T *out, const RealGeom &g,
               const Cx<T> *twM, const int *skip, hipStream_t st, hipError_t &err)
 {
+    auto one = [&](auto n1, auto n2) {
+        err = launch_x_one<T, n1, n2, WRAP>(forward, data, in, out, g, twM, skip, st);
+        return true;
+    };
     switch (M) {
-    case 176: err = launch_x_one<T, 16, 11>(forward, data, in, out, g, twM, skip, st); return true;
-    case 192: err = launch_x_one<T, 16, 12>(forward, data, in, out, g, twM, skip, st); return true;
-    case 256: err = launch_x_one<T, 16, 16>(forward, data, in, out, g, twM, skip, st); return true;
-    case 320: err = launch_x_one<T, 20, 16>(forward, data, in, out, g, twM, skip, st); return true;
-    case 360: err = launch_x_one<T, 20, 18>(forward, data, in, out, g, twM, skip, st); return true;
-    case 384: err = launch_x_one<T, 24, 16>(forward, data, in, out, g, twM, skip, st); return true;
-    case 448: err = launch_x_one<T, 28, 16>(forward, data, in, out, g, twM, skip, st); return true;
-    case 512: err = launch_x_one<T, 32, 16>(forward, data, in, out, g, twM, skip, st); return true;
-    case 640: err = launch_x_one<T, 32, 20>(forward, data, in, out, g, twM, skip, st); return true;
+    case 176: return one(Len<16>{}, Len<11>{});
+    case 192: return one(Len<16>{}, Len<12>{});
+    case 256: return one(Len<16>{}, Len<16>{});
+    case 320: return one(Len<20>{}, Len<16>{});
+    case 360: return one(Len<20>{}, Len<18>{});
+    case 384: return one(Len<24>{}, Len<16>{});
+    case 448: return one(Len<28>{}, Len<16>{});
+    case 512: return one(Len<32>{}, Len<16>{});
+    case 640: return one(Len<32>{}, Len<20>{});
     default: return false;
     }
 }
