@@ -788,15 +788,18 @@ int make_axis(AxisPlan &ap, size_t M, const char *what);
 // The y pass over planes [k0, k0 + nk) of the half spectrum in the
 // register form (fft_reg.h), when M1 has a split: forward reads rows
 // [lo, hi) and stores every row; inverse reads every row and stores rows
-// [lo, hi).  False: no split, nothing launched.
-template <typename T>
+// [lo, hi).  WRAP (forward): both ranges may wrap.  False: no split, nothing
+// launched.
+template <typename T, bool WRAP = false>
 bool y_reg(Cx<T> *work, const Vol &v, int k0, int nk, const AxisPlan &ap, bool forward, int lo,
            int hi, const int *skip, hipStream_t st, hipError_t &err)
 {
     reg::PenGeom pg;
     pg.H = v.M0;
     pg.npen = v.M0 * nk;
-    pg.base0 = size_t(k0) * v.M0 * v.M1;
+    pg.base0 = WRAP ? 0 : size_t(k0) * v.M0 * v.M1;
+    pg.r0 = k0;
+    pg.nr = v.M2;
     pg.rstep = size_t(v.M0) * v.M1;
     pg.istride = size_t(v.M0);
     pg.lo_in = forward ? lo : 0;
@@ -804,10 +807,14 @@ bool y_reg(Cx<T> *work, const Vol &v, int k0, int nk, const AxisPlan &ap, bool f
     pg.lo_out = forward ? 0 : lo;
     pg.hi_out = forward ? v.M1 : hi;
     const reg::NoOp<T> none;
-    return forward
-        ? reg::launch<T, reg::FWD>(v.M1, work, work, pg, twM_of<T>(ap), none, skip, st, err)
-        : reg::launch<T, reg::LOAD_K | reg::INV>(v.M1, work, work, pg, twM_of<T>(ap), none,
-                                                 skip, st, err);
+    if constexpr (WRAP)
+        return reg::launch<T, reg::FWD | reg::WRAP>(v.M1, work, work, pg, twM_of<T>(ap), none,
+                                                    skip, st, err);
+    else
+        return forward
+            ? reg::launch<T, reg::FWD>(v.M1, work, work, pg, twM_of<T>(ap), none, skip, st, err)
+            : reg::launch<T, reg::LOAD_K | reg::INV>(v.M1, work, work, pg, twM_of<T>(ap), none,
+                                                     skip, st, err);
 }
 
 // The z pass in the register form, when M2 has a split: pencils (x, y) of
@@ -821,6 +828,8 @@ bool z_reg(Cx<T> *dst, const Cx<T> *src, const Vol &v, const AxisPlan &ap, int z
     pg.H = v.M0;
     pg.npen = v.M0 * v.M1;
     pg.base0 = 0;
+    pg.r0 = 0;
+    pg.nr = v.M1;
     pg.rstep = size_t(v.M0);
     pg.istride = size_t(v.M0) * v.M1;
     pg.lo_in = zlo;
@@ -904,9 +913,8 @@ int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const 
             work, in, g, pn, ap[0].dpl, tw_of<T>(ap[0]), skip);
         QSM_HIP(hipGetLastError());
     }
-    // y forward on data planes (the register-resident y and z passes take no
-    // range that wraps)
-    if (!WRAP && y_reg<T>(work, v, g.o2, nz, ap[1], true, g.o1, g.o1 + ny, skip, st, e)) {
+    // y forward on data planes
+    if (y_reg<T, WRAP>(work, v, g.o2, nz, ap[1], true, g.o1, g.o1 + ny, skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pny = pencils(M1, cs);
@@ -916,8 +924,9 @@ int real_conv(const T *in, T *out, const size_t sz[3], const size_t M[3], const 
         QSM_HIP(hipGetLastError());
     }
     // z forward, op (, z inverse)
-    constexpr int ZM = ROUND ? (reg::FWD | reg::OP | reg::INV) : (reg::FWD | reg::OP);
-    if (!WRAP && z_reg<T, ZM>(work, work, v, ap[2], g.o2, g.o2 + nz, op, skip, st, e)) {
+    constexpr int ZM = ROUND ? (reg::FWD | reg::OP | reg::INV)
+                             : (reg::FWD | reg::OP | (WRAP ? reg::WRAP : 0));
+    if (z_reg<T, ZM>(work, work, v, ap[2], g.o2, g.o2 + nz, op, skip, st, e)) {
         QSM_HIP(e);
     } else {
         const Pen pn = pencils(M2, cs);

@@ -181,13 +181,15 @@ struct PenGeom {
     size_t base0, rstep, istride;
     int lo_in, hi_in;    // n-order loads: elements outside are zero, not read
     int lo_out, hi_out;  // n-order stores: elements outside are not written
+    int r0, nr;          // WRAP: pencil row r stands at wrap(r0 + r, nr)
 };
 
 // What a pass does, in order: load (n order, or k order with LOAD_K),
 // forward transform (FWD, n -> k order), op(x, r, k, value) on every sample
 // (OP), inverse transform (INV, k -> n order), store (k order: every
-// element; n order: [lo_out, hi_out)).
-enum : int { LOAD_K = 1, FWD = 2, OP = 4, INV = 8 };
+// element; n order: [lo_out, hi_out)).  WRAP: [lo_in, hi_in) and the pencil
+// rows may run past the axis's end and go on at 0.
+enum : int { LOAD_K = 1, FWD = 2, OP = 4, INV = 8, WRAP = 16 };
 
 template <int N1, int N2>
 constexpr int team() { return N1 > N2 ? N1 : N2; }
@@ -200,7 +202,9 @@ __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void pen4(
     constexpr int M = N1 * N2, TM = team<N1, N2>(), NT = P * TM;
     constexpr bool kin = (MODE & LOAD_K) != 0, fwd = (MODE & FWD) != 0;
     constexpr bool useop = (MODE & OP) != 0, inv = (MODE & INV) != 0;
+    constexpr bool wraps = (MODE & WRAP) != 0;
     static_assert(kin != fwd, "a pass loads in n order exactly when it transforms forward");
+    static_assert(!wraps || !inv, "n-order stores take no range that wraps");
     __shared__ Cx<T> X[P * M];
     __shared__ Cx<T> W[M];
     if (skip && *skip)
@@ -208,7 +212,8 @@ __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void pen4(
     const int t = int(threadIdx.x), p = t % P, m = t / P;
     const int q = xcd_block() * P + p;
     const bool live = q < g.npen;
-    const int x = live ? q % g.H : 0, r = live ? q / g.H : 0;
+    const int x = live ? q % g.H : 0, rq = live ? q / g.H : 0;
+    const int r = wraps ? wrap<true>(g.r0 + rq, g.nr) : rq;
     const Cx<T> *in = src + (g.base0 + size_t(x) + size_t(r) * g.rstep);
     Cx<T> *out = dst + (g.base0 + size_t(x) + size_t(r) * g.rstep);
     const size_t is = g.istride;
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(P * (N1 > N2 ? N1 : N2)) void pen4(
                 constexpr int n1 = decltype(c)::value;
                 const int i = N2 * n1 + m;
                 a[n1] = Cx<T>{T(0), T(0)};
-                if (live && i >= g.lo_in && i < g.hi_in)
+                if (live && in_range<wraps>(i, g.lo_in, g.hi_in, M))
                     a[n1] = in[size_t(i) * is];
             });
         }

@@ -164,3 +164,15 @@ def test_ball_wraps_around_sample_zero(cuda, shape, vsz, r, dt):
     gf, gm = gbg.vsharp(f, m, vsz, rs)
     np.testing.assert_array_equal(gm, wm)
     assert rel_l2(gf, wf) < (1e-10 if dt == np.float64 else 1e-4)
+
+
+# The register-resident y and z passes take the ball's range that wraps: both
+# axes of a register length, a short range on either side of sample 0 and one
+# nearly as long as the axis (161 of 176 and of 192 rows and planes).
+@pytest.mark.parametrize("shape,vsz,r", [((6, 168, 184), (1.0, 1.0, 1.0), 4.0),
+                                         ((5, 184, 168), (1.0, 2.0, 1.3), 4.0),
+                                         ((16, 32, 16), (0.5, 0.5, 0.5), 40.0),
+                                         ((32, 16, 32), (1.0, 1.0, 1.0), 80.0)])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_ball_wraps_in_the_register_passes(cuda, shape, vsz, r, dt):
+    test_ball_wraps_around_sample_zero(cuda, shape, vsz, r, dt)
