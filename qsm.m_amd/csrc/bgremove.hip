@@ -62,6 +62,7 @@ __global__ __launch_bounds__(NT) void ball_kernel(T *h, int M0, int R1, int R2, 
     h[l] = ((Y * Y + X * X) + Z * Z <= r2) ? v : T(0);
 }
 
+// The SMV multipliers at half-spectrum sample (x, y, z), from Sb = 2
 // FFT3(ifftshift(ball)) as the x pass leaves it (H = Sb.re / 2 in the class
 // Tb of f: real(fft3(ifftshift(h))), sharp.m:62):
 //   MODE 0  H                (the mask smoothing, sharp.m:63)
