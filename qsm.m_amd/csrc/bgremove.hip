@@ -165,7 +165,7 @@ size_t ball_reach(const double vsz[3], double r, int axis)
 // spectra (V-SHARP keeps the first radius's for its deconvolution), the
 // convolution's work spectrum, the spectra of the mask and of a single
 // echo's f that V-SHARP reuses for every radius, two float volumes and two
-// of the class of f on the crop, three byte masks.  The two reused spectra
+// of the class of f on the crop, two byte masks.  The two reused spectra
 // are laid out only for the calls that use them (SPEC_* bits): SHARP needs
 // neither, multi-echo V-SHARP only the mask's.
 template <typename T>
@@ -175,7 +175,7 @@ struct Work {
     Cx<float> *Sm;
     float *mf, *sf;
     T *g, *c;
-    uint8_t *m1, *mp, *mo;
+    uint8_t *m1, *mp;
 };
 
 enum { SPEC_F = 1, SPEC_M = 2 };
@@ -197,7 +197,7 @@ size_t layout(const size_t szc[3], const size_t M[3], const double vsz[3], doubl
     char *psm = (spectra & SPEC_M) ? take(real_conv_work_bytes(M, sizeof(float))) : nullptr;
     char *pmf = take(n * sizeof(float)), *pvf = take(n * sizeof(float));
     char *pg = take(n * sizeof(T)), *pc = take(n * sizeof(T));
-    char *pm1 = take(n), *pmp = take(n), *pmo = take(n);
+    char *pm1 = take(n), *pmp = take(n);
     if (w) {
         w->ball = reinterpret_cast<T *>(pb);
         w->Sb = reinterpret_cast<Cx<T> *>(ps);
@@ -211,7 +211,6 @@ size_t layout(const size_t szc[3], const size_t M[3], const double vsz[3], doubl
         w->c = reinterpret_cast<T *>(pc);
         w->m1 = reinterpret_cast<uint8_t *>(pm1);
         w->mp = reinterpret_cast<uint8_t *>(pmp);
-        w->mo = reinterpret_cast<uint8_t *>(pmo);
     }
     return off;
 }
@@ -230,7 +229,7 @@ void plan_for(const size_t szc[3], const double vsz[3], double rmax, size_t M[3]
 // wrap around sample 0 (361 of 44100 rows and 19 of 175 planes for r = 9 at
 // 216x252x175, where forming and transforming all of them took 89 us more
 // per radius, of about 115).  The padding of rmax on either side makes an
-// axis longer than its ball.
+// axis longer than its ball, which reaches at least one row and plane.
 template <typename T>
 int ball_spectrum(Cx<T> *Sb, T *ball, const size_t M[3], const double vsz[3], double r,
                   hipStream_t st)
@@ -242,7 +241,7 @@ int ball_spectrum(Cx<T> *Sb, T *ball, const size_t M[3], const double vsz[3], do
     ball_kernel<T><<<grid1(sz[0] * sz[1] * sz[2]), NT, 0, st>>>(
         ball, int(M[0]), int(R1), int(R2), vsz[0], vsz[1], vsz[2], r * r, T(1.0 / double(K)));
     QSM_HIP(hipGetLastError());
-    const size_t off[3] = {0, R1 > 0 ? M[1] - R1 : 0, R2 > 0 ? M[2] - R2 : 0};
+    const size_t off[3] = {0, M[1] - R1, M[2] - R2};
     return real_conv<T, false, true>(ball, static_cast<T *>(nullptr), sz, M, off, Sb, KeepOp<T>{},
                                      st);
 }
@@ -342,9 +341,9 @@ int vsharp_t(const T *fc, const uint8_t *mc, const size_t szc[3], size_t nech,
     if (one && (rc = real_conv<T, false>(fc, static_cast<T *>(nullptr), szc, M, off, w.Sf,
                                          KeepOp<T>{}, st)))
         return rc;
-    // the masks of this radius, of the last one and of the one returned, in
-    // three buffers that change places
-    uint8_t *cur = w.m1, *prev = w.mp, *spare = w.mo, *ret = nullptr;
+    // the masks of this radius and of the last one, in two buffers that change
+    // places; the one returned is one of the two that the loop leaves
+    uint8_t *cur = w.m1, *prev = w.mp, *ret = nullptr;
     for (size_t q = 0; q < nrs; ++q) {
         Cx<T> *Sb = q == 0 ? w.Sb1 : w.Sb;  // the first radius's spectrum is kept for ih
         if ((rc = ball_spectrum<T>(Sb, w.ball, M, vsz, rs[q], st))) return rc;
@@ -364,10 +363,7 @@ int vsharp_t(const T *fc, const uint8_t *mc, const size_t szc[3], size_t nech,
             }
         }
         if (q == qout) ret = cur;
-        // the buffer of the radius before last is free, unless it is returned
-        uint8_t *freed = prev == ret ? spare : prev;
-        prev = cur;
-        cur = freed;
+        std::swap(cur, prev);
     }
     // f = maskn .* real(ifft3(ih .* fft3(f))), ih from the first radius,
     // maskn the last radius's mask (vsharp.m:142-143)

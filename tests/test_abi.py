@@ -163,15 +163,15 @@ def test_sharp_work_bytes_only_hold_what_each_call_uses():
 def test_sharp_work_bytes_hold_the_ball_on_its_rows(szc, vsz, r, grid, dt, es):
     """The ball image takes its own rows and planes of the transform grid,
     whole in x, not the grid; besides it three spectra, two float volumes,
-    two of the class of f and three masks, each rounded up to 256 bytes."""
+    two of the class of f and two masks, each rounded up to 256 bytes."""
     from qsm_amd import bgremove as bg
 
     n = szc[0] * szc[1] * szc[2]
     ball = grid[0] * (2 * math.ceil(r / vsz[1]) + 1) * (2 * math.ceil(r / vsz[2]) + 1)
     assert ball < grid[0] * grid[1] * grid[2]
     spec = (grid[0] // 2 + 1) * grid[1] * grid[2] * 2 * es
-    lo = ball * es + 3 * spec + 2 * 4 * n + 2 * es * n + 3 * n
-    assert lo <= bg.work_bytes(dt, szc, vsz, r) <= lo + 11 * 255
+    lo = ball * es + 3 * spec + 2 * 4 * n + 2 * es * n + 2 * n
+    assert lo <= bg.work_bytes(dt, szc, vsz, r) <= lo + 10 * 255
 
 
 @pytest.mark.parametrize("rmax,vsz", [(float("nan"), (1, 1, 1)), (-3.0, (1, 1, 1)), (0.0, (1, 1, 1)),
