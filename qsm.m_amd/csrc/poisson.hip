@@ -632,18 +632,22 @@ dim3 cheb_grid(Dim d)
     return dim3((d.nx - 2 + CB - 1) / CB, (d.ny - 2 + CB - 1) / CB, (d.nz - 2 + CB - 1) / CB);
 }
 
-// Whether a level takes boxes: those that the chip's 256 CUs hold at once,
-// two per CU in FP32 (32 KB of LDS each) and one in FP64 (64 KB: two fit, but
-// then each takes twice as long).  Solves of one level, one PCG iteration,
-// boxes against one step per launch, MI355X: FP32 0.67 / 0.76 ms at 512 boxes
-// (64x64x64), 0.90 / 0.83 at 648 (72x72x64), 2.76 / 1.46 at 4096 (256x256x30);
-// FP64 0.57 / 0.63 ms at 245 (56x56x40), 0.77 / 0.69 at 294 (56x56x48), 0.94 /
-// 0.97 at 512, 4.59 / 2.75 at 4096.
+// Whether a level takes boxes.  The chip's 256 CUs hold two each (32 KB of LDS
+// in FP32, 64 KB in FP64), 512 at once; more need a second round and lose.  In
+// FP64 two on a CU take twice as long as one, so the time of boxes doubles at
+// 257 and then stands, while that of a step per launch grows with the level:
+// they meet again at about 380.  Solves of one level, one PCG iteration, boxes
+// against one step per launch, MI355X: FP32 0.64 / 0.71 ms at 512 boxes
+// (64x64x64), 0.79 / 0.72 at 576 (66x64x64), 2.76 / 1.46 at 4096 (256x256x30);
+// FP64 0.51 / 0.58 ms at 256 (64x64x32), 0.68 / 0.59 at 288 (64x72x32), 0.72 /
+// 0.68 at 360 (72x64x40), 0.78 / 0.81 at 384 (64x64x48), 0.91 / 0.95 at 512,
+// 1.14 / 0.95 at 576, 4.59 / 2.75 at 4096.
 template <typename T>
 bool cheb_boxed(Dim d)
 {
     const dim3 g = cheb_grid(d);
-    return size_t(g.x) * g.y * g.z <= (sizeof(T) == 4 ? 512 : 256);
+    const size_t n = size_t(g.x) * g.y * g.z;
+    return n <= 512 && (sizeof(T) == 4 || n <= 256 || n >= 384);
 }
 
 struct ChebSteps {

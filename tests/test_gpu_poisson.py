@@ -279,15 +279,15 @@ def test_unwrap_work_space_at_any_address(cuda, dt):
 
 
 # One-level solves on either side of the lines between the coarsest level's
-# two kernels (512 boxes of 8^3 in FP32, 256 in FP64), the grid's rows and
+# two kernels (512 boxes of 8^3; in FP64 256, 384 and 512), the grid's rows and
 # planes in each place, rows that end within a group of four.  The Chebyshev
 # polynomial maps the spectrum of the operator into 1 +- 1e-3 whatever the
 # mask, so PCG's bound is 2 (5e-4)^k in the energy norm and, with the square
 # root of the condition number below 100, 200 (5e-4)^k in the residual: 5
 # iterations for 1e-12, 3 for 1e-5, one more for rounding.
-@pytest.mark.parametrize("shape", [(128, 128, 1), (129, 128, 1), (128, 256, 1), (129, 256, 1),
-                                   (2, 127, 259), (127, 259, 2), (259, 2, 127), (18, 131, 137),
-                                   (64, 62, 63), (66, 67, 65)])
+@pytest.mark.parametrize("shape", [(128, 128, 1), (129, 128, 1), (136, 176, 1), (128, 192, 1),
+                                   (128, 256, 1), (129, 256, 1), (2, 127, 259), (127, 259, 2),
+                                   (259, 2, 127), (18, 131, 137), (64, 62, 63), (66, 67, 65)])
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_mgpcg_coarsest_level_sizes(cuda, shape, dt):
     rng = np.random.default_rng(shape[0])
