@@ -128,17 +128,30 @@ def test_mgpcg_argument_checks_without_gpu(kw, msg):
     assert e.value.code == _lib.QSM_EARG
 
 
-def test_mgpcg_work_bytes_cover_the_hierarchy():
-    """Work space: per level v, f, r and two mask bytes, and on the levels
-    that smooth (all but the coarsest) the band's index lists (n + 1 ints);
-    PCG x, p; coarse CG scratch; band seed; the lists' per-row counts
-    (2 ints per level-0 row); reduction partials."""
-    n = [(34, 30, 26), (18, 16, 14), (10, 9, 8)]      # 32x28x24 padded, 3 levels
-    vox = [a * b * c for a, b, c in n]
-    w = _lib.lib().qsm_mgpcg_work_bytes(_lib.F64, (C.c_size_t * 3)(32, 28, 24), 3)
-    lo = (sum(3 * 8 * v + 2 * v for v in vox) + sum(4 * (v + 1) for v in vox[:-1])
-          + 2 * 8 * vox[0] + 2 * 8 * vox[-1] + vox[0] + 2 * 4 * n[0][1] * n[0][2])
-    assert lo <= w <= lo + 64 * 1024
+@pytest.mark.parametrize("sz,levels,cheb", [((32, 28, 24), 3, 4),      # coarsest level in boxes
+                                            ((129, 128, 1), 1, 3),     # one step per launch
+                                            ((1, 5, 7), 1, 4)])
+@pytest.mark.parametrize("dt,es", [(_lib.F64, 8), (_lib.F32, 4)])
+def test_mgpcg_work_bytes_cover_the_hierarchy(sz, levels, cheb, dt, es):
+    """Work space, fields kept by colour with half rows of a multiple of four
+    positions: per level v, f and two mask bytes, and on the levels that smooth
+    (all but the coarsest) the band's index lists (a word per voxel and one);
+    PCG x, p; the coarsest level's d twice and r, twice where boxes update it
+    (the one-step form takes over earlier in FP64); band seed and two levels'
+    masks in natural order; the lists' per-row counts (2 ints per level-0
+    row); reduction partials."""
+    dims = [tuple(s + 2 for s in sz)]
+    for _ in range(levels - 1):
+        dims.append(tuple(((s - 1) >> 1) + 2 for s in dims[-1]))
+    nat = [a * b * c for a, b, c in dims]
+    pos = [2 * (((a + 1) // 2 + 3) // 4 * 4) * b * c for a, b, c in dims]
+    if dt == _lib.F32:
+        cheb = 4
+    w = _lib.lib().qsm_mgpcg_work_bytes(dt, (C.c_size_t * 3)(*sz), levels)
+    lo = (sum(2 * es * n + 2 * n for n in pos) + sum(4 * (n + 1) for n in nat[:-1])
+          + 2 * es * pos[0] + cheb * es * pos[-1] + 2 * nat[0] + (nat[1] if levels > 1 else 0)
+          + 2 * 4 * dims[0][1] * dims[0][2] + 1024 * 8)
+    assert lo <= w <= lo + 8 * 1024
 
 
 def test_sharp_work_bytes_only_hold_what_each_call_uses():
